@@ -558,7 +558,7 @@ int tfa_prefill_attention(const void* q, int64_t q_rs, int64_t q_hs, const void*
 /* C[m, n] = bf16(A[m, k] . B[n, k]^T) (residual == NULL) or
  * C = bf16(residual + bf16(A . B^T)) (residual [m, ldr]); bf16 in, f32 accumulate
  * on bf16 MFMA, the residual added in the kernel's epilogue. Row strides lda /
- * ldb / ldc in elements. m >= 1, n a multiple of 128, k of 64; lda, ldb
+ * ldb / ldc in elements, below 2^31 (here and in every product below). m >= 1, n a multiple of 128, k of 64; lda, ldb
  * multiples of 8, ldc, ldr of 4; a, b 16-byte and c, residual 8-byte aligned.
  * Replaces: examples/qwen3_8_27b_prefill-tilelang/kernels/gemm.py:104-356 (gemm_kernel,
  * "residual" epilogue :193-198 -- model.py:326-333 Attention.o_proj). */

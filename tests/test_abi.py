@@ -177,6 +177,10 @@ def test_prompt_prefill_argument_checks(lib):
     assert st == SHAPE
     st, _ = call(lib, "tfa_gemm_nt_f32", P(None), A, A, I64(37), I64(512), I64(2048), I64(2048), I64(2048), I64(512), P(None))
     assert st == NULL
+    # row pitches past 31 bits (a single row has none)
+    for lda, ldb, ldc in ((1 << 31, 2048, 512), (2048, 1 << 31, 512), (2048, 2048, 1 << 31)):
+        st, msg = call(lib, "tfa_gemm_nt_f32", A, A, A, I64(37), I64(512), I64(2048), I64(lda), I64(ldb), I64(ldc), P(None))
+        assert st == SHAPE and "pitch" in msg
     # split f32 GEMM: splits that do not divide the k-tiles, too many splits
     st, msg = call(lib, "tfa_gemm_nt_f32_split", A, A, A, I64(37), I64(512), I64(2048), I64(2048), I64(2048),
                    I64(512), I64(3), P(None))

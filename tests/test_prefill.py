@@ -202,6 +202,70 @@ def test_gemm_tile_edges_exact(dev, M, N, K):
     assert_equal("residual", out, (res.float() + ref.to(BF).float()).to(BF))
 
 
+def _pitched(rows: torch.Tensor, ld: int) -> torch.Tensor:
+    """The rows as a view ``ld`` elements apart (the room between is never touched)."""
+    m, k = rows.shape
+    out = torch.empty((m - 1) * ld + k, dtype=rows.dtype, device=rows.device).as_strided((m, k), (ld, 1))
+    out.copy_(rows)
+    return out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("wide,ld", [("a", 2 ** 27 - 8), ("a", 2 ** 27), ("a", 2 ** 28 + 64), ("b", 2 ** 27)])
+@pytest.mark.parametrize("M,K", [(17, 64), (19, 320)])
+def test_gemm_wide_pitches(dev, M, K, wide, ld):
+    """Row pitches at and past 2^27 elements, where 16 rows span 2^32 bytes, against the
+    same rows packed: every store and epilogue, one k-tile and five, K in ranges.
+    Integer inputs, exact in f32, so every element is equal."""
+    from tilefoundry_amd._lib import C
+
+    if torch.cuda.mem_get_info()[0] < 40 << 30:
+        pytest.skip("needs 33 GiB of address room for 128 rows of 2^27 elements")
+    N = 128
+    g = torch.Generator().manual_seed(M + K)
+    a = torch.randint(-3, 4, (M, K), generator=g).to(BF).to(dev)
+    b = torch.randint(-3, 4, (N, K), generator=g).to(BF).to(dev)
+    res = torch.randint(-8, 9, (M, N), generator=g).to(BF).to(dev)
+    gamma, (cos, sin) = torch.ones(128, device=dev, dtype=BF), (torch.rand(M, 128, device=dev).to(BF) for _ in range(2))
+
+    def every(a, b):
+        out = {"f32": torch.empty(M, N, device=dev), "part": torch.empty(K // 64, M, N, device=dev)}
+        out |= {n: torch.empty(M, w, device=dev, dtype=BF) for n, w in (("plain", N), ("res", N), ("act", N // 2), ("q", N))}
+        C.gemm_nt_f32(a, b, out["f32"])
+        C.gemm_nt_f32(a, b, out["part"])
+        C.gemm_nt(a, b, out["plain"], None)
+        C.gemm_nt(a, b, out["res"], res)
+        C.gemm_nt_swiglu(a, b, out["act"])
+        # three heads of the same 128 weight rows
+        if wide == "a":
+            kc = torch.zeros(M, 128, device=dev, dtype=BF)
+            out["k"], out["v"] = kc, kc.clone()
+            C.gemm_nt_qk_rope(a, b.repeat(3, 1), gamma, gamma, 1e-6, cos, sin, 1, M, 0, kc, out["v"], out["q"], 1, 1)
+        else:
+            out.pop("q")
+        return out
+
+    far = every(_pitched(a, ld) if wide == "a" else a, _pitched(b, ld) if wide == "b" else b)
+    near = every(a, b)
+    assert_equal("f32 product", near["f32"], a.float().cpu() @ b.float().cpu().t())
+    for name in near:
+        assert_equal(name, far[name], near[name])
+    torch.cuda.empty_cache()
+
+
+@pytest.mark.gpu
+def test_gemm_single_row_has_no_pitch(dev):
+    """One row of A and C: whatever pitch the view states, it is not used."""
+    from tilefoundry_amd._lib import C
+
+    g = torch.Generator().manual_seed(3)
+    a = torch.randint(-3, 4, (1, 128), generator=g).to(BF).to(dev)
+    b = torch.randint(-3, 4, (256, 128), generator=g).to(BF).to(dev)
+    out = torch.empty(1, 256, dtype=BF, device=dev)
+    C.gemm_nt(a.as_strided((1, 128), (2 ** 33, 1)), b, out.as_strided((1, 256), (2 ** 33, 1)), None)
+    assert_equal("single row", out, (a.float().cpu() @ b.float().cpu().t()).to(BF))
+
+
 def _layer_weights(seed=5):
     return OP.random_layer(CFG, seed=seed)
 

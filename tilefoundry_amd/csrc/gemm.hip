@@ -165,7 +165,7 @@ using C128 = Cfg<128, 128, 2, 2>;      // 4 waves of 64 x 64, two blocks per CU
 
 constexpr int kWaitVm0 = waitcnt_vm(0);
 
-template <class C, int EPI>
+template <class C, int EPI, bool WIDE>
 __global__ __launch_bounds__(C::kThreads) void gemm_kernel(const GemmArgs a) {
   constexpr int BM = C::BM, BN = C::BN, TI = C::kTI, TJ = C::kTJ;
   __shared__ __attribute__((aligned(1024))) uint16_t smem[C::kSmem];
@@ -196,7 +196,9 @@ __global__ __launch_bounds__(C::kThreads) void gemm_kernel(const GemmArgs a) {
   // k-tile is a scalar offset. Rows past M lie past the descriptor's end and come
   // as zeros (never stored); so does every row of a k-tile past the last one, whose
   // load is issued against an empty descriptor and moves nothing -- the k loop's
-  // body and its wait counts are the same to the end.
+  // body and its wait counts are the same to the end. WIDE (row pitches whose 16
+  // rows a 32-bit descriptor does not span): a 64-bit address per lane instead, with
+  // rows past M reading row M - 1 and k-tiles past the last one the last again.
   constexpr int kHA = C::kWTM / 2, kHB = C::kWTN / 2;        // rows of one wave's half
   constexpr int kGA = BM / 16 / C::kWaves, kGB = BN / 16 / C::kWaves, kGD = kGA + kGB;   // loads per wave and group
   static_assert(kGA >= 1 && kGB >= 1 && kHA % (8 * kGA) == 0 && kHB % (8 * kGB) == 0 && kHA % 16 == 0 && kHB % 16 == 0,
@@ -204,11 +206,12 @@ __global__ __launch_bounds__(C::kThreads) void gemm_kernel(const GemmArgs a) {
   static_assert(kGD * 2 * 8 * C::kWaves == C::kRows, "two groups fill a stage");
   i32x4 rsrc[2][2];                 // [group][A, B]
   uint32_t voff[kGD], dst[kGD];     // lane offsets (both groups); LDS byte offsets of group 0
+  const char* wsrc[WIDE ? 2 : 1][WIDE ? kGD : 1];
   {
     const int ra = 8 * kGA * wid, rb = 8 * kGB * wid;
     const int rowa = ra / kHA * C::kWTM + ra % kHA, rowb = rb / kHB * C::kWTN + rb % kHB;   // stage rows of group 0
 #pragma unroll
-    for (int g = 0; g < 2; ++g) {
+    for (int g = 0; g < 2 && !WIDE; ++g) {
       const int first = min(m0 + rowa + g * kHA, a.M - 1);
       rsrc[g][0] = buffer_of(a.a + static_cast<size_t>(first) * a.lda, 2u * a.lda * min(a.M - first, 8 * kGA));
       rsrc[g][1] = buffer_of(a.b + static_cast<size_t>(n0 + rowb + g * kHB) * a.ldb, 2u * a.ldb * (8 * kGB));
@@ -218,12 +221,23 @@ __global__ __launch_bounds__(C::kThreads) void gemm_kernel(const GemmArgs a) {
     for (int i = 0; i < kGD; ++i) {
       const bool isa = i < kGA;
       const int j = 8 * (isa ? i : i - kGA), row = (isa ? rowa : rowb) + j;
-      voff[i] = 2u * ((j + l3) * (isa ? a.lda : a.ldb) + 8 * ((lane & 7) ^ swz(row + l3)));
+      const int chunk = 8 * ((lane & 7) ^ swz(row + l3));   // the same in both groups
       dst[i] = lds_offset(&smem[((isa ? 0 : BM) + row) * kBK]);
+      if constexpr (WIDE) {
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+          const int r = row + g * (isa ? kHA : kHB) + l3;
+          wsrc[g][i] = reinterpret_cast<const char*>(
+              (isa ? a.a + static_cast<size_t>(min(m0 + r, a.M - 1)) * a.lda : a.b + static_cast<size_t>(n0 + r) * a.ldb) + chunk);
+        }
+      } else {
+        voff[i] = 2u * ((j + l3) * (isa ? a.lda : a.ldb) + chunk);
+      }
     }
   }
   // k-tile kt's scalar offset; past the last k-tile the descriptors are emptied
   auto at_tile = [&](int kt) __attribute__((always_inline)) {
+    if constexpr (WIDE) return static_cast<uint32_t>((kt0 + min(kt, nk - 1)) * (kBK * 2));
     const int keep = kt < nk ? -1 : 0;
 #pragma unroll
     for (int g = 0; g < 2; ++g)
@@ -234,8 +248,12 @@ __global__ __launch_bounds__(C::kThreads) void gemm_kernel(const GemmArgs a) {
   // load i of group g into stage st
   auto dma1 = [&](int g, int i, uint32_t soff, int st) __attribute__((always_inline)) {
     const uint32_t half = (i < kGA ? kHA : kHB) * kBK * 2;
-    asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff[i]), "s"(rsrc[g][i < kGA ? 0 : 1]), "s"(soff),
-                 "{m0}"(dst[i] + g * half + st * C::kStage * 2) : "memory");
+    const uint32_t to = dst[i] + g * half + st * C::kStage * 2;
+    if constexpr (WIDE)
+      lds_dma16(wsrc[g][i] + soff, to);
+    else
+      asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff[i]), "s"(rsrc[g][i < kGA ? 0 : 1]), "s"(soff),
+                   "{m0}"(to) : "memory");
   };
   auto dma = [&](int g, uint32_t kt, int st) __attribute__((always_inline)) {
 #pragma unroll
@@ -558,11 +576,11 @@ __global__ __launch_bounds__(C::kThreads) void gemm_kernel(const GemmArgs a) {
   }
 }
 
-template <class C, int EPI>
+template <class C, int EPI, bool WIDE = false>
 int launch_cfg(const GemmArgs& g, hipStream_t st, const char* name) {
   const int nm = (g.M + C::BM - 1) / C::BM, nn = g.N / C::BN;
   const unsigned splits = EPI == EPI_F32 && g.ksplit > 1 ? (unsigned)g.ksplit : 1u;
-  gemm_kernel<C, EPI><<<dim3((unsigned)(nm * nn), splits), C::kThreads, 0, st>>>(g);
+  gemm_kernel<C, EPI, WIDE><<<dim3((unsigned)(nm * nn), splits), C::kThreads, 0, st>>>(g);
   return launched(name);
 }
 
@@ -642,9 +660,16 @@ int pick_tile(int64_t m, int64_t n, int cus) {
   return c128x256 <= c128 ? TILE_128x256 : TILE_128;
 }
 
+// Row pitch (elements) from which a wave's 16 stage rows no longer fit a 32-bit
+// descriptor: 16 rows * 2 bytes * 2^27 = 2^32, and the lane offsets wrap with it.
+constexpr int kWidePitch = 1 << 27;
+
 template <int EPI>
 int launch(const GemmArgs& g, hipStream_t st, const char* name) {
   const int cus = device_cus();
+  if constexpr (EPI != EPI_QKNR) {   // (its operands are contiguous, at most 2^24 wide)
+    if (g.lda >= kWidePitch || g.ldb >= kWidePitch) return launch_cfg<C128, EPI, true>(g, st, name);
+  }
   if constexpr (EPI == EPI_QKNR) {
     // Whole 256-column head slices: 256 or 128 rows, by rounds of one block per CU. A
     // 128-row round takes two thirds of a 256-row one (the weights' half of the
@@ -675,6 +700,8 @@ int check_gemm(const void* a, const void* b, const void* c, int64_t m, int64_t n
                 (long long)m, (long long)n, (long long)k);
   if (lda < k || ldb < k || ldc < n || lda % 8 || ldb % 8 || ldc % 4)
     return fail(TFA_ERR_SHAPE, "%s: leading dimensions too small, or lda / ldb not multiples of 8, ldc of 4", fn);
+  if (ldb > INT32_MAX || (m > 1 && (lda > INT32_MAX || ldc > INT32_MAX)))   // a single row has no pitch
+    return fail(TFA_ERR_SHAPE, "%s: row pitches of 2^31 elements and more are not supported", fn);
   if (!aligned16(a) || !aligned16(b)) return fail(TFA_ERR_ALIGN, "%s: a / b not 16-byte aligned", fn);
   if ((reinterpret_cast<uintptr_t>(c) & 7u) != 0) return fail(TFA_ERR_ALIGN, "%s: c not 8-byte aligned", fn);
   return TFA_OK;
@@ -685,7 +712,8 @@ GemmArgs make(const void* a, const void* b, int64_t m, int64_t n, int64_t k, int
   g.a = static_cast<const uint16_t*>(a);
   g.b = static_cast<const uint16_t*>(b);
   g.M = (int)m; g.N = (int)n; g.K = (int)k;
-  g.lda = (int)lda; g.ldb = (int)ldb; g.ldc = (int)ldc;
+  g.lda = (int)(m == 1 ? k : lda);   // a single row has no pitch
+  g.ldb = (int)ldb; g.ldc = (int)ldc;
   return g;
 }
 
@@ -700,8 +728,8 @@ int tfa_gemm_nt(const void* a, const void* b, void* c, int64_t m, int64_t n, int
   GemmArgs g = make(a, b, m, n, k, lda, ldb, ldc);
   g.c = static_cast<uint16_t*>(c);
   if (residual) {
-    TFA_REQUIRE(ldr >= n && ldr % 4 == 0, TFA_ERR_SHAPE, "tfa_gemm_nt: ldr %lld < n %lld or not a multiple of 4",
-                (long long)ldr, (long long)n);
+    TFA_REQUIRE(ldr >= n && ldr % 4 == 0 && (m == 1 || ldr <= INT32_MAX), TFA_ERR_SHAPE,
+                "tfa_gemm_nt: ldr %lld < n %lld, not a multiple of 4 or past 2^31", (long long)ldr, (long long)n);
     TFA_REQUIRE((reinterpret_cast<uintptr_t>(residual) & 7u) == 0, TFA_ERR_ALIGN,
                 "tfa_gemm_nt: residual not 8-byte aligned");
     g.res = static_cast<const uint16_t*>(residual);
@@ -737,8 +765,8 @@ int tfa_gemm_nt_swiglu(const void* a, const void* b, void* act, int64_t m, int64
                        int64_t ldb, int64_t ldact, hipStream_t stream) {
   const int st = check_gemm(a, b, act, m, n, k, lda, ldb, n, "tfa_gemm_nt_swiglu");
   if (st != TFA_OK) return st;
-  TFA_REQUIRE(ldact >= n / 2 && ldact % 2 == 0, TFA_ERR_SHAPE,
-              "tfa_gemm_nt_swiglu: ldact %lld below n / 2 = %lld or odd", (long long)ldact, (long long)(n / 2));
+  TFA_REQUIRE(ldact >= n / 2 && ldact % 2 == 0 && (m == 1 || ldact <= INT32_MAX), TFA_ERR_SHAPE,
+              "tfa_gemm_nt_swiglu: ldact %lld below n / 2 = %lld, odd or past 2^31", (long long)ldact, (long long)(n / 2));
   GemmArgs g = make(a, b, m, n, k, lda, ldb, ldact);
   g.c = static_cast<uint16_t*>(act);
   return launch<EPI_SWIGLU>(g, stream, "gemm_nt_swiglu");
