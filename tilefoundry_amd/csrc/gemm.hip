@@ -88,16 +88,6 @@ TFA_DEV i32x4 buffer_of(const void* p, uint32_t bytes) {
 typedef uint32_t u32x4a8 __attribute__((ext_vector_type(4), aligned(8)));
 typedef uint32_t u32x2a4 __attribute__((ext_vector_type(2), aligned(4)));
 
-// x / (1 + e^-x) with the hardware's exponential and reciprocal: within 2^-20 of
-// the quotient for |x| < 16, so a landed bf16 result differs from the divided one's
-// only that close to a rounding boundary. Below -87 (e^-x past 2^126, where
-// the reciprocal would be subnormal) the quotient is formed by scaling.
-TFA_DEV float silu_fast(float x) {
-  const float d = 1.0f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f);
-  const float r = __builtin_amdgcn_rcpf(d);
-  return d > 0x1p126f ? x * __builtin_amdgcn_rcpf(d * 0x1p-24f) * 0x1p-24f : x * r;
-}
-
 TFA_DEV bf16x8 as_bf8(uint4 v) { return __builtin_bit_cast(bf16x8, v); }
 
 enum { EPI_STORE = 0, EPI_RESID = 1, EPI_F32 = 2, EPI_QKNR = 3, EPI_SWIGLU = 4, EPI_QKROPE = 5 };
@@ -435,11 +425,15 @@ __global__ __launch_bounds__(C::kThreads) void gemm_kernel(const GemmArgs a) {
       if (grow >= a.M) return;
       u32x4 v = *reinterpret_cast<const u32x4*>(ep + row * C::kEpPitch + cl);
       if constexpr (EPI == EPI_SWIGLU) {
-        // columns 2 i, 2 i + 1 are gate and up of output i; the decode step's order:
+        // columns 2 i, 2 i + 1 are gate and up of output i; the decode step's order and
+        // its divided silu, so a prompt row lands as the same token decoded does:
         // bf16(bf16(silu(bf16 g)) * bf16 u)
         float y[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) y[i] = round_bf(silu_fast(lo_bf(v[i]))) * hi_bf(v[i]);
+        for (int i = 0; i < 4; ++i) {
+          const float x = lo_bf(v[i]);
+          y[i] = round_bf(x / (1.0f + expf(-x))) * hi_bf(v[i]);
+        }
         *reinterpret_cast<u32x2a4*>(a.c + static_cast<size_t>(grow) * a.ldc + (n0 + cl) / 2) =
             u32x2a4{pack_bf(y[0], y[1]), pack_bf(y[2], y[3])};
       } else {
