@@ -231,6 +231,10 @@ def prefill_caches(cfg: Qwen3Config, embed, layers, kc, vc, cos, sin, ids: torch
         k4 = kc[i].view(B, -1, HKV, D)
         v4 = vc[i].view(B, -1, HKV, D)
         k3, v3 = k4.view(B, -1, HKV * D), v4.view(B, -1, HKV * D)
+        if part["qkv"] is None and any(t.data_ptr() % 8 for t in (w["gamma_q"], w["gamma_k"], cos, sin, k3, v3)):
+            # the epilogue reads and writes these 8 bytes at a time; the separate
+            # launch, from here on, takes them at any alignment
+            part["qkv"] = e(C.gemm_f32_splits(R, *shapes["qkv"]), R, cfg.qkv_rows, dtype=f32)
         if part["qkv"] is None:
             C.gemm_nt_qk_rope(xn, w["w_qkv"], w["gamma_q"], w["gamma_k"], cfg.eps, cos, sin, B, n, 0, k3, v3, q, HQ, HKV)
         else:
