@@ -527,6 +527,17 @@ def test_mla_block_vs_reference(dev, B, cap, pos, fuse_qb):
         assert_l2(f"o_proj b={b}", branch, ref.float() @ ow.w_o.float().t())
 
 
+def test_folds_only_what_the_split_form_takes():
+    """The folded launches take no plan that the split product or the consumer of its
+    partials refuses: ranges of whole steps, at least one and at most eight."""
+    from tilefoundry_amd.minicpm3 import _folds
+
+    assert _folds(2560, 5, 3072, 256) and _folds(2560, 1, 3072, 256) and _folds(2048, 8, 3072, 256)
+    assert not _folds(2560, 10, 3072, 256)   # ten ranges: the residual sums at most eight
+    assert not _folds(2560, 0, 3072, 256) and not _folds(2560, 3, 3072, 256)
+    assert not _folds(3584, 7, 3072, 256) and not _folds(2304, 1, 3072, 256)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,n,k", [(1, 16, 512), (8, 2560, 2560), (15, 24, 1024), (16, 272, 1536), (17, 2560, 2560), (32, 40, 3072)])
 def test_skinny_gemm_scaled_residual_exact(dev, m, n, k):

@@ -138,8 +138,9 @@ def rope_tables(n: int, cfg: MiniCPM3Config, device):
 
 def _folds(k: int, ks: int, most: int, unit: int) -> bool:
     """Whether a projection of depth ``k`` planned as ``ks`` ranges may run with its
-    neighbour folded in: what the split form refuses stays with it and is refused."""
-    return ks >= 1 and k <= most and k % 512 == 0 and k % (unit * ks) == 0
+    neighbour folded in: what the split form or the consumer of its partials (at most
+    8 ranges) refuses stays with them and is refused."""
+    return 1 <= ks <= 8 and k <= most and k % 512 == 0 and k % (unit * ks) == 0
 
 
 class MLABlock:
