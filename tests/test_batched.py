@@ -509,6 +509,16 @@ def test_batch_engine_attention_choice():
     assert pick(8, 64) and not pick(8, 128) and not pick(48, 1536)
 
 
+def test_batch_engine_prep_choice():
+    """The query prep runs in the split attention's blocks only where those are few:
+    not from 64 pairs up, and not over a cache whose grid has more than 4096 blocks."""
+    from tilefoundry_amd.qwen3 import BatchEngine
+
+    pick = BatchEngine._prep_in_blocks
+    assert pick(8, 512) and not pick(8, 513) and pick(56, 64) and not pick(56, 256)
+    assert pick(63, 1) and not pick(64, 1)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("batch", [1, 3, 7])
 def test_batch_engine_split_prep_forms(dev, batch, monkeypatch):

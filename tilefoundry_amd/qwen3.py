@@ -551,10 +551,11 @@ class BatchEngine:
         batch_sample     greedy step per sequence
 
     With fewer blocks than that (``attention="split"``) the attention is split-KV
-    ``decode_attention`` and ``attn_combine``: from 64 (sequence, kv head) pairs up
-    with ``qk_rope_cache`` before it (the query prepared once per sequence), below
-    that with the prep in the attention's own blocks. ``"auto"`` picks between the
-    two forms by pairs and cache (``_whole_context``).
+    ``decode_attention`` and ``attn_combine``: from 64 (sequence, kv head) pairs up,
+    and over long caches, with ``qk_rope_cache`` before it (the query prepared once per
+    sequence), else with the prep in the attention's own blocks (``_prep_in_blocks``).
+    ``"auto"`` picks between whole-context and split by pairs and cache
+    (``_whole_context``).
     """
 
     MAX_BATCH = 32
@@ -603,8 +604,21 @@ class BatchEngine:
         if capture:
             self._capture()
 
-    #: pairs (sequences x kv heads) from which a launch for the query prep alone pays
+    #: pairs (sequences x kv heads) from which a launch for the query prep alone pays, and
+    #: blocks of the split grid (pairs x splits of the whole cache) past which it pays below that
     PREP_PAIRS = 64
+    PREP_BLOCKS = 4096
+
+    @classmethod
+    def _prep_in_blocks(cls, pairs: int, splits: int) -> bool:
+        """Whether the split attention's own blocks prepare the query. It saves a launch,
+        but every block of the grid loads its heads, those past the context too. Steps of
+        four layers, launch against blocks, us: 6 sequences x 8 heads in a cache of 3072
+        198 / 194 at 380 positions, 217 / 207 at 1500; 7 in 8192 (3,584 blocks) 223 / 218
+        at 1000, 332 / 329 at 8100; 2 in 32768 (4,096) 194 / 196 at 1500, 355 / 354 at
+        32000; 4 in 32768 (8,192) 219 / 228 at 1500, 284 / 290 at 8000; 7 in 32768
+        (14,336) 237 / 264 and 348 / 371. At 16 sequences the two are equal."""
+        return pairs < cls.PREP_PAIRS and pairs * splits <= cls.PREP_BLOCKS
 
     @staticmethod
     def _whole_context(pairs: int, cap: int) -> bool:
@@ -666,9 +680,8 @@ class BatchEngine:
                 C.decode_attention_seq(self.qkv_part, w["gamma_q"], w["gamma_k"], cfg.eps, self.cos, self.sin,
                                        self.pos, self.pos, self.kc[i], self.vc[i], HQ, HKV, cfg.scale, self.attn,
                                        self.err)
-            elif self.batch * HKV < self.PREP_PAIRS:
+            elif self._prep_in_blocks(self.batch * HKV, self.ns):
                 # few blocks: the prep in each of them costs less than its launch
-                # (a step of four layers at 6 x 1500: 212 against 221 us; at 16, equal)
                 C.decode_attention(None, self.qkv_part, w["gamma_q"], w["gamma_k"], cfg.eps, self.cos, self.sin,
                                    self.kc[i], self.vc[i], self.pos, self.pos, HQ, HKV, self.split, cfg.scale,
                                    self.op, self.mp, self.lp, False, self.err)
