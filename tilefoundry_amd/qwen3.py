@@ -625,12 +625,16 @@ class BatchEngine:
         """Whether one block per (sequence, kv head) over its whole context beats the
         splits for a cache of ``cap`` positions. It saves two launches and the
         partials (10-12 us a layer), but below one pair per CU a long context runs on
-        too few of them. Steps of four layers, splits against whole context, us: 6
-        sequences x 8 heads 190 / 183 at 20 positions, 212 / 250 at 1500; 12: 206 / 187
-        at 20, 220 / 219 at 600, 244 / 259 at 1500; 16: 216 / 193 at 200, 266 / 263 at
-        1500, 319 / 350 at 3000; 24: 239 / 203 at 200, 389 / 389 at 3000; 31: 258 / 213
-        at 200, 459 / 427 at 3000. A sequence passes through every context up to the
-        cache, so the line is where half the cache breaks even."""
+        too few of them. Steps of four layers, splits against whole context, us: 2
+        sequences x 8 heads 179 / 175 at 60 positions, 178 / 190 at 340; 3: 180 / 178 and
+        181 / 190; 4 in a cache of 256 183 / 179 at 128, 183 / 180 at 200, in 512 183 / 193
+        at 256; 5: 185 / 180, 185 / 181 and 184 / 194; 6: 190 / 183 at 20, 212 / 250 at
+        1500; 8: 193 / 183 at 128, 194 / 196 at 256; 12: 206 / 187 at 20, 223 / 223 at 768,
+        240 / 251 at 1476; 16: 216 / 193 at 200, 266 / 263-272 at 1500, 319 / 350 at 3000;
+        20: 282 / 257 at 1152, 335 / 332 at 2304, 440 / 459 at 4548; 24: 239 / 203 at 200,
+        389 / 389 at 3000, 594 / 606 at 6200; 31: 258 / 213 at 200, 599 / 549 at 4544. A
+        sequence passes through every context up to the cache, so the line is where half
+        the cache breaks even."""
         return pairs >= 256 or cap <= max(8 * pairs, 50 * (pairs - 66))
 
     def _buffers(self):
