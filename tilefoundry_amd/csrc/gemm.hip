@@ -628,30 +628,35 @@ bool fused_epilogue(int64_t m, int64_t n, int64_t k) {
   return (m + 127) / 128 * (n / 128) * 4 >= kSplitPlanCus * 3;
 }
 
-// Tile choice of the bf16 stores. Blocks run in rounds, one per CU (two of the
-// 128 x 128 tile), so the time is the rounds times what one takes. In units of a
-// 256 x 256 round (62 us at K = 2048, 145 at 6144): a 128 x 256 round 56, a 128 x 128
-// round 57 with two blocks on every CU, 62 with two on some and 42 with one.
-// Measured, us, 256 x 256 / 128 x 256 / 128 x 128: 12288 x 2048 at 509 rows 52.7 / 36.5 /
-// 41.1, at 1500 108.7 / 97.3 / 87.3, at 4000 190.9 / 208.8 / 206.3; 5120 x 6144 at 640
-// rows 50 with 128 x 128 (200 blocks), at 1024 95 with it (320) and 75 with 128 x 256
-// (160), at 2048 136 with 128 x 128. A half-empty last round of a long grid costs
-// less than a whole one (the card is at its power limit), so from two rounds on
-// 256 x 256 may lose by 8 % on paper: 5120 x 6144 at 8192 rows (2.5 rounds) takes
-// 442 with it, 474 with 128 x 128.
+// Tile choice of the bf16 stores: the least of three costs, in hundredths of a full
+// round of 256 x 256 tiles (62 us at 12288 x 2048, 105 at 8192 x 4096, 155 at 5120 x
+// 6144). Blocks run in rounds, one per CU (two of the 128 x 128 tile). A first round
+// waits for weights out of HBM whatever it holds, so a part-filled round of large tiles
+// costs most of a full one; later rounds overlap the one before and a nearly empty last
+// one adds a third. Fitted to six shapes at 36 row counts each over uncached weights
+// (with cached ones a round of 128 x 256 looks as cheap as 50 of 5120 x 6144's 75 us, and
+// 101 is what it takes): the tile picked is within 5 % of the best at all of them.
+// Examples, us, 256 x 256 / 128 x 256 / 128 x 128: 5120 x 6144 at 640
+// rows 121 / 103 / 69, 896 121 / 102 / 94, 1152 117 / 101 / 114, 1664 130 / 159 / 153, 4608
+// 277 / 270 / 305, 8192 452 / 511 / 541; 12288 x 2048 with SwiGLU at 509 51 / 36 / 40, 1500
+// 106 / 95 / 85, 4000 186 / 207 / 205; 8192 x 4096 at 1280 88 / 111 / 99.
 enum { TILE_256, TILE_128x256, TILE_128 };
 
-int pick_tile(int64_t m, int64_t n, int cus) {
+int pick_tile(int64_t m, int64_t n, int64_t k, int cus) {
   if (n % 256) return TILE_128;
-  auto rounds = [&](int64_t blocks) { return (blocks + cus - 1) / cus; };
-  const int64_t b128 = (m + 127) / 128 * (n / 128);
-  const int64_t rest = b128 % (2 * cus);
-  const int64_t c128 = b128 / (2 * cus) * 57 + (rest == 0 ? 0 : rest <= cus ? 42 : 62);
-  const int64_t c128x256 = 56 * rounds((m + 127) / 128 * (n / 256));
-  const int64_t r256 = rounds((m + 255) / 256 * (n / 256));
-  const int64_t best = c128x256 <= c128 ? c128x256 : c128;
-  if (r256 * 100 <= best || (r256 >= 2 && r256 * 100 * 100 <= best * 108)) return TILE_256;
-  return c128x256 <= c128 ? TILE_128x256 : TILE_128;
+  const int64_t rows128 = (m + 127) / 128;
+  const int64_t b256 = (m + 255) / 256 * (n / 256), bx = rows128 * (n / 256), b128 = rows128 * (n / 128);
+  const int64_t l256 = b256 % cus, lx = bx % cus, l128 = b128 % (2 * cus);   // blocks of the last, part-filled round
+  const int64_t c256 = b256 / cus * 100 + (l256 ? 71 + 21 * l256 / cus : 0);
+  // (a lone round over a long K is a little dearer: 288 blocks of 128 x 128 take 94 us of 6144
+  // where 144 take 102, 35.5 of 2048 where 144 take 33)
+  const int64_t cx = bx <= cus ? (k > 4096 ? 66 : 65) : 65 + (bx / cus - 1) * 54 + (lx ? 30 + 18 * lx / cus : 0);
+  auto two = [&](int one, int both, int more) -> int64_t {   // up to one block on each CU, or two on some
+    return l128 == 0 ? 0 : l128 <= cus ? one : both + more * (l128 - cus) / cus;
+  };
+  const int64_t c128 = b128 < 2 * cus ? two(46, 64, 8) : 72 + (b128 / (2 * cus) - 1) * 57 + two(20, 50, 17);
+  if (c256 <= cx && c256 <= c128) return TILE_256;
+  return cx <= c128 ? TILE_128x256 : TILE_128;
 }
 
 // Row pitch (elements) from which a wave's 16 stage rows no longer fit a 32-bit
@@ -678,7 +683,7 @@ int launch(const GemmArgs& g, hipStream_t st, const char* name) {
     return full_rounds_256(g.M, g.N, cus) && g.ksplit == 1 ? launch_cfg<C256, EPI>(g, st, name)
                                                             : launch_cfg<C128, EPI>(g, st, name);
   } else {
-    switch (pick_tile(g.M, g.N, cus)) {
+    switch (pick_tile(g.M, g.N, g.K, cus)) {
       case TILE_256: return launch_cfg<C256, EPI>(g, st, name);
       case TILE_128x256: return launch_cfg<C128x256, EPI>(g, st, name);
       default: return launch_cfg<C128, EPI>(g, st, name);
