@@ -503,7 +503,8 @@ void launch_trw(const SkinnyArgs& a, hipStream_t st) {
     constexpr bool kHead = EPI == SK_ARGMAX || EPI == SK_ARGMAX_BF16;
     if (NP == NP_OWN || (a.M <= 16 && !(kHead && a.M <= kFewTokens))) return go(std::integral_constant<int, 1>{});
   }
-  if constexpr (NP == NP_NONE && (EPI == SK_PARTIAL || EPI == SK_SWIGLU)) {   // prompt rows
+  // prompt rows: tfa_prompt_gemm alone, whose K ranges of whole 512-element steps run eight waves
+  if constexpr (W == 8 && NP == NP_NONE && (EPI == SK_PARTIAL || EPI == SK_SWIGLU)) {
     if (a.M > 48) return go(std::integral_constant<int, 4>{});
     if (a.M > 32) return go(std::integral_constant<int, 3>{});
   }
@@ -1010,7 +1011,7 @@ int tfa_skinny_gemm(const void* x, const void* w, int64_t m, int64_t n, int64_t 
 // 16 / 61 rows: 4096 x 2048 9.8 -> 8.4 / 10.8 -> 10.4, 12288 x 2048 with SwiGLU 16.7 -> 11.5 /
 // 18.2 -> 14.5, 2048 x 2048 9.9 -> 7.2 / 11.3 -> 9.0, 2048 x 6144 14.9 -> 10.0 / 16.9 -> 13.1.
 int64_t tfa_prompt_gemm_splits(int64_t m, int64_t n, int64_t k) {
-  if (m < 1 || m > kMaxPromptRows || n < 1 || k < kWaves * kChunk) return 0;
+  if (m < 1 || m > kMaxPromptRows || n < 1 || k < 1) return 0;
   // as many K ranges as give every CU a block of 32 weight rows, of whole 512-element
   // steps (eight waves), at most four: the partials go through memory
   int64_t ks = 1;
