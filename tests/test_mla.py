@@ -527,6 +527,25 @@ def test_mla_block_vs_reference(dev, B, cap, pos, fuse_qb):
         assert_l2(f"o_proj b={b}", branch, ref.float() @ ow.w_o.float().t())
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("ks_o", [2, 5])
+def test_block_o_proj_partials(dev, ks_o):
+    """``part_o`` holds the split o_proj product of the last step in every slice, also
+    where the step itself runs the projection unsplit with its residual."""
+    from tilefoundry_amd._lib import C
+    from tilefoundry_amd.minicpm3 import MLABlock, MiniCPM3Config, synthetic_weights
+
+    cfg = MiniCPM3Config()
+    wts = synthetic_weights(cfg, seed=7)
+    blk = MLABlock(cfg, batch=2, cap=256, device=dev, weights=wts, ks_o=ks_o)
+    hidden = torch.randn(2, cfg.hidden, generator=gen(3)).to(BF).to(dev)
+    for pos in ([0, 9], [1, 10]):   # each step's own
+        blk.step(hidden, pos)
+        ref = torch.empty(ks_o, 2, cfg.hidden, device=dev)
+        C.skinny_gemm(blk.attn, blk.w["w_o"], ks_o, 0, ref, None, None, None, None)
+        assert torch.equal(blk.part_o, ref)
+
+
 def test_folds_only_what_the_split_form_takes():
     """The folded launches take no plan that the split product or the consumer of its
     partials refuses: ranges of whole steps, at least one and at most eight."""

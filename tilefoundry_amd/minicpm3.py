@@ -176,7 +176,7 @@ class MLABlock:
 
         self.ns = cap // split
         self.hidden = z(B, cfg.hidden)
-        self.xn = z(B, cfg.hidden)
+        self.xn = None if self.fold_norm else z(B, cfg.hidden)
         self.part_a = z(ks_a, B, cfg.q_lora + cfg.kv_lora + cfg.rope, dtype=f32)
         self.q_n = z(B, cfg.q_lora)
         self.part_qb = z(ks_qb, B, H * cfg.qk_dim, dtype=f32)
@@ -187,7 +187,7 @@ class MLABlock:
         self.mp = z(B, self.ns, H, dtype=f32)
         self.lp = z(B, self.ns, H, dtype=f32)
         self.attn = z(B, H * cfg.v_dim)
-        self.part_o = z(ks_o, B, cfg.hidden, dtype=f32)
+        self._part_o = z(ks_o, B, cfg.hidden, dtype=f32)
         self.out = z(B, cfg.hidden)
         self.pos = z(B, dtype=torch.int32)
         self.err = z(1, dtype=torch.int32)
@@ -212,11 +212,19 @@ class MLABlock:
                         self.op, self.mp, self.lp, self.err)
         C.mla_combine_up(self.op, self.mp, self.lp, self.pos, self.split, w["w_kv_b"], self.attn)
         if self.fold_o:
-            # part_o: the unrounded product in its first slice, the others stay zero
-            C.skinny_gemm_scaled_residual(self.attn, w["w_o"], self.hidden, self.alpha, self.out, self.part_o[0])
+            C.skinny_gemm_scaled_residual(self.attn, w["w_o"], self.hidden, self.alpha, self.out, None)
         else:
-            C.skinny_gemm(self.attn, w["w_o"], self.ks["o"], 0, self.part_o, None, None, None, None)
-            C.rows_residual(self.part_o, self.hidden, self.alpha, self.out)
+            C.skinny_gemm(self.attn, w["w_o"], self.ks["o"], 0, self._part_o, None, None, None, None)
+            C.rows_residual(self._part_o, self.hidden, self.alpha, self.out)
+
+    @property
+    def part_o(self) -> torch.Tensor:
+        """The last step's o_proj before its residual, f32 split-K partials ``[ks_o, batch,
+        hidden]``. Where the residual is folded into the projection no step needs them,
+        and they are computed here, from ``attn``."""
+        if self.fold_o:
+            C.skinny_gemm(self.attn, self.w["w_o"], self.ks["o"], 0, self._part_o, None, None, None, None)
+        return self._part_o
 
     def capture(self):
         """Record one step as a graph (inputs: ``hidden``, ``pos``, the caches)."""
