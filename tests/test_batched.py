@@ -227,12 +227,12 @@ def test_skinny_own_norm_swiglu(dev, M, N, K):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,V,K", [(5, 65553, 2048), (16, 65553, 2560), (17, 32785, 1024), (32, 32785, 1536), (32, 40000, 2048),
-                                   (17, 32785, 2560), (32, 40001, 2560)])
+@pytest.mark.parametrize("M,V,K", [(1, 65553, 2048), (5, 65553, 2048), (9, 65553, 2560), (10, 65553, 2560), (16, 65553, 2560),
+                                   (17, 32785, 1024), (32, 32785, 1536), (32, 40000, 2048), (17, 32785, 2560), (32, 40001, 2560)])
 @pytest.mark.parametrize("epilogue", [2, 3])   # argmax of the f32 values / of the bf16 ones
 def test_skinny_head_walk_is_the_plain_head(dev, M, V, K, epilogue):
-    """A vocabulary of many row tiles is walked by one block per CU: the same bits as
-    its slices, which a block per tile computes."""
+    """A vocabulary of many row tiles is walked by one block per CU (2560 wide from ten
+    tokens on): the same bits as its slices, which a block per tile computes."""
     from tilefoundry_amd._lib import C
     g = gen(V + M)
     x = randn(M, K, g=g).to(dev)

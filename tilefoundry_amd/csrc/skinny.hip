@@ -46,7 +46,8 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kWaves = 4;
 constexpr int kMaxTokens = 32;
-constexpr int kFewTokens = 4;    // the head keeps the plain form with two token tiles
+constexpr int kFewTokens = 4;    // the plain head keeps two token tiles
+constexpr int kWalkTokens5 = 10; // from here on a head of five chunks is walked
 constexpr int kMaxPromptRows = 64;
 constexpr int kGroupRows = 16;   // argmax winners are kept per 16 weight rows
 
@@ -498,8 +499,9 @@ void launch_trw(const SkinnyArgs& a, hipStream_t st) {
       skinny_gemm_kernel<EPI, 1, TR, W, TM, NP><<<grid, W * kWave, 0, st>>>(a);
   };
   if constexpr (NP != NP_SSQ && EPI != SK_RESID_SSQ) {
-    // (the head of up to four tokens reads as fast with two: 54.9 us in a MiniCPM3 step of one
-    // sequence, its walk 55.8)
+    // (up to four tokens the head reads a little faster with two, one / two us: 73448 x 2560
+    // 55.2 / 54.8 at 1, 56.8 / 56.3 at 4, 57.2 / 57.4 at 6, 59.3 / 59.8 at 8; 131072 x 2560
+    // 95.5 / 94.8, 97.0 / 96.3 at 4, 98.3 / 99.5 at 8; 65536 x 2560 equal up to 4)
     constexpr bool kHead = EPI == SK_ARGMAX || EPI == SK_ARGMAX_BF16;
     if (NP == NP_OWN || (a.M <= 16 && !(kHead && a.M <= kFewTokens))) return go(std::integral_constant<int, 1>{});
   }
@@ -522,18 +524,22 @@ void launch_tr(const SkinnyArgs& a, hipStream_t st) {
 }
 
 // The head's walk: from four tiles a CU where it saves the second token tile's reads
-// too; up to 16 tokens the saving is half, and it takes the loads of four chunks a wave
-// and eight tiles a CU to beat two resident blocks. Plain / walk, us, over rotating
-// weights: 151936 x 2048 at 1 / 16 / 32 tokens 98.2/96.9, 104.3/100.6, 122.9/106.0 (with
-// logits 32: 134.4/112.8 = 5.7 TB/s), 73448 x 2560 59.1/59.1, 63.9/60.7, 77.5/65.5, 32800 x
-// 2048 at 17 / 32 29.3/26.4, 31.4/27.9. Left to the plain form: 32800 x 2048 at 16
-// 24.1/25.1, 128001 x 1024 at 1 41.7/44.5, and up to four tokens, where nothing is saved.
+// too; up to 16 tokens the saving is half, and it takes eight tiles a CU and the loads of
+// four chunks a wave to beat two resident blocks. Plain / walk, us, over rotating weights:
+// 151936 x 2048 at 1 / 4 / 8 / 16 / 32 tokens 99.0/93.5, 98.6/94.3, 100.0/96.5, 105.4/100.1,
+// 122.9/106.0 (with logits 32: 134.4/112.8 = 5.7 TB/s), 65536 x 2048 at 1 / 4 / 16 45.5/42.9,
+// 45.5/43.4, 46.9/45.4, 32800 x 2048 at 17 / 32 29.3/26.4, 31.4/27.9. With five chunks it pays
+// from ten tokens on: 73448 x 2560 with logits at 1 / 4 / 8 / 9 / 10 / 16 54.8/55.3, 56.3/57.0,
+// 59.3/58.7, 59.8/59.9, 62.3/60.8, 70.6/63.4, 131072 x 2560 94.8/96.4 at 1, with logits
+// 104.5/109.0, 105.4/107.0, 108.8/108.3 at 8 / 9 / 10. Left to the plain form besides: 32800 x
+// 2048 at 16 24.1/25.1, 128001 x 1024 at 1 41.7/44.5. Five chunks are the most: two token
+// tiles hold 32 registers a chunk, 232 in all at five.
 template <int EPI>
 bool launch_head(const SkinnyArgs& a, hipStream_t st) {
   const int cus = skinny_cus(), tiles = (a.N + 31) / 32, nc = a.K / (8 * kChunk);
   if (a.K % (8 * kChunk) || nc < 2 || nc > 5 || tiles < 4 * cus) return false;
   if (a.M <= 16) {
-    if (a.M <= kFewTokens || nc < 4 || tiles < 8 * cus) return false;
+    if (nc < 4 || (nc > 4 && a.M < kWalkTokens5) || tiles < 8 * cus) return false;
     if (nc == 4)
       skinny_head_kernel<EPI, 4, 1><<<cus, 8 * kWave, 0, st>>>(a);
     else
