@@ -36,14 +36,15 @@
 // then stage loads), and the two barriers of a k-tile stand where the operands of
 // the phase after them are already in registers. What bounds it: at full grids
 // the power limit -- on random data 1.16-1.34 PFLOP/s (8192 x 14336 x 5120, plain
-// store 895 us, with the head-norm epilogue 960), on all-zero data 1.64 (734 us)
+// store 891 us, with the head-norm epilogue 901), on all-zero data 1.64 (734 us, 746)
 // -- before that the LDS port, whose operand reads and stage writes take as many
 // cycles as the MFMAs. One barrier and a full wait per k-tile, with the first
-// reads behind it, took 1,040 us where this takes 960, and 64 us where this takes
-// 50 (640 x 5120 x 6144 + residual, 200 blocks of 128 x 128: one per CU, so
-// nothing else hides the waits). Also measured: 4 waves of 128 x 128 (a quarter
-// less LDS traffic, but one wave per SIMD) 1,030 us; stage loads in a burst
-// behind each barrier 986 us.
+// reads behind it, took 1,040 us with the head norm where this took 960 (901 since
+// the epilogue's sixteen lanes to a head row), and 64 us where this takes 50 (640 x
+// 5120 x 6144 + residual with cached weights, 200 blocks of 128 x 128: one per CU, so
+// nothing else hides the waits). Also measured, beside the 960: 4 waves of 128 x 128
+// (a quarter less LDS traffic, but one wave per SIMD) 1,030 us; stage loads in a
+// burst behind each barrier 986 us.
 //
 // Epilogue (bf16 outputs): the tile lands in bf16 into LDS (rows padded by 32
 // bytes), then each wave takes whole rows -- 16 bytes per lane for the store, the
@@ -617,7 +618,7 @@ int64_t splits_f32(int64_t m, int64_t n, int64_t k) {
 // but with fewer 128 x 128 blocks than CUs it cannot draw the weights from HBM as
 // fast as a split grid. Measured over weights not in any cache, split + consumer
 // against fused, us: 12288 x 2048 (SwiGLU) 26.0 / 27.6 at 128 rows (96 blocks),
-// 29.3 / 25.4 at 200 (192), 50.3 / 36.5 at 509, 497 / 372 at 8000; 4096 x 2048
+// 28.2 / 24.4 at 200 (192), 50.4 / 34.9 at 509, 493 / 356 at 8000; 4096 x 2048
 // (norm, RoPE, cache rows) 29.0 / 28.5 at 509 (128), 33.2 / 28.4 at 700 (192), 214 /
 // 146 at 8000; 2048 x 2048 (residual, norm) 25.7 / 26.9 at 999 (128), 31.8 / 27.9 at
 // 1500 (192); 2048 x 6144 45.3 / 67.1 at 999, 66.8 / 67.3 at 1500, 71.1 / 67.0 at 2000

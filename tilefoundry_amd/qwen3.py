@@ -181,7 +181,7 @@ def prefill_caches(cfg: Qwen3Config, embed, layers, kc, vc, cos, sin, ids: torch
     ``swiglu_pairs`` -- lands the sums as the decode step lands its split-K
     partials. The attention of every row is one causal launch over the cache
     (``causal_attention``). Only the summation order of the products differs from
-    the walk. 7 to 11 launches per layer, none per token; the last layer stops
+    the walk. 7 to 9 launches per layer, none per token; the last layer stops
     after its cache rows (nothing downstream of them reaches a cache).
 
     This replaces the reference's token-by-token prompt walk
@@ -199,14 +199,14 @@ def prefill_caches(cfg: Qwen3Config, embed, layers, kc, vc, cos, sin, ids: torch
 
     h, h1, xn = e(R, H), e(R, H), e(R, H)
     shapes = {"qkv": (cfg.qkv_rows, H), "o": (H, HQ * D), "gu": (2 * I, H), "down": (H, I)}
-    # f32 split-K partials [ks, R, out] of the projections that run split; the
-    # consumers sum them in split order, as the decode step sums its own
     # few rows run on the decode step's skinny product, which keeps more of the
     # weights in flight than a 128-row tile does: a layer's four projections and
     # their consumers at 61 rows 57 -> 47 us, at 16 rows 51 -> 37
     splits = {name: C.prompt_gemm_splits(R, *s) for name, s in shapes.items()}
     short = all(splits.values()) and all(
         w[k].is_contiguous() for w in layers for k in ("w_qkv", "w_o", "w_gu", "w_down"))
+    # f32 split-K partials [ks, R, out] of the projections that run split; the
+    # consumers sum them in split order, as the decode step sums its own
     if short:
         part = {name: e(splits[name], R, s[0], dtype=f32) for name, s in shapes.items() if name != "gu"}
     else:
